@@ -222,9 +222,8 @@ int hs_batch_stats(const hs_ctx* ctx, uint64_t* batch_calls, uint64_t* graph_cap
 /* Tile choices of the step kernels (no reference counterpart; the reference
  * fixes one strand per invocation in workgroups of 32, compute.comp:4,13, and
  * Renderer.cpp:2070).  Results are identical for every choice; only the speed
- * changes.  One lane steps one strand (64 strands per wavefront); the
- * workgroup takes `strands` strands and walks them root to tip `points`
- * points at a time.  (strands, points) is one of the built shapes: (128, 16),
+ * changes.  A workgroup takes `strands` strands and walks them root to tip
+ * `points` points at a time.  (strands, points) is one of the built shapes: (128, 16),
  * (256, 8), (256, 12).  A change of shape takes effect on the next step. */
 typedef struct hs_tile {
     uint32_t gather_cells;  /* voxels of the LDS window the friction gather stages, 64..2048 */
@@ -292,9 +291,9 @@ int hs_grid_near_limit(hs_ctx* ctx, uint32_t groom_id, uint64_t* cells);
  * workgroup-segment's own box goes to a slot of its own and is not
  * counted) with the shared capacities, whether anything fell back to device
  * atomics (a box larger than any LDS window, or a full pool), and how many
- * workgroup-segments had a box larger than one window and were splatted
- * chunk by chunk by the workgroups that finished first.  Zeros before the
- * first such step.  Blocks. */
+ * workgroup-segments had a box larger than one window (splatted window by
+ * window, or with device atomics when that takes more than 32).  Zeros before
+ * the first such step.  Blocks. */
 typedef struct hs_grid_work_stats {
     uint32_t pool_cells, pool_capacity, boxes, box_capacity, fallback, deferred;
 } hs_grid_work_stats;

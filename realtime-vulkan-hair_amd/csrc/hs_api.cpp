@@ -93,13 +93,9 @@ uint64_t carve(Groom& g, uint8_t* base)
         take(g.gw.brick_list, bricks(g.G) * 2 * hs::kBrickList * 4);
         take(g.gw.brick_nz, bricks(g.G) * 4);  // zero: every brick of the zeroed grid is empty
         take(g.gw.near_limit, 8);
-        take(g.gw.dlist, 2ull * L.nws_cap * 8);
-        take(g.gw.dclaim, 2ull * L.nws_cap * 4);
-        take(g.gw.dbox, (uint64_t)L.nws_cap * hs::kDBoxInts * 4);
         g.gw.pool_cap = (uint32_t)L.pool_cap;
         g.gw.desc_cap = (uint32_t)L.desc_cap;
         g.gw.nws = L.nws_cap;  // each launch sets its tile shape's count
-        g.gw.nws_cap = L.nws_cap;
         g.gw.nbx = bricks_x(g.G);
         g.gw.nby = bricks_y(g.G);
         g.gw.nbz = bricks_z(g.G);
@@ -344,7 +340,6 @@ int build_args(hs_ctx* c, Groom& g, const hs_time* t, const hs_collider* cols, u
     a.gbox_ok = g.last_shape == c->shape ? 1u : 0u;
     a.G = g.G;
     a.parity = g.parity;
-    a.tag = g.steps % 0x0fffffffu + 1u;  // 28 bits, never 0: the deferred list starts zero-filled
     a.ox = g.origin[0];
     a.oy = g.origin[1];
     a.oz = g.origin[2];
@@ -409,7 +404,6 @@ int build_args(hs_ctx* c, Groom& g, const hs_time* t, const hs_collider* cols, u
 // the tile shape its boxes were written in.
 void advance_state(Groom& g, bool splat, float friction, int shape)
 {
-    g.steps += 1;
     if (splat) {
         g.last_shape = shape;
         g.parity ^= 1u;
@@ -1363,7 +1357,7 @@ int hs_grid_work(hs_ctx* c, uint32_t id, hs_grid_work_stats* out)
     out->pool_capacity = g->gw.pool_cap - g->gw.nws * hs::kSlotCells;
     out->boxes = ctr[1];
     out->box_capacity = g->gw.desc_cap - g->gw.nws;
-    out->fallback = ctr[2];
+    out->fallback = ctr[2] & hs::kFellBack;
     out->deferred = ctr[3];
     return HS_OK;
 }

@@ -52,25 +52,6 @@ __device__ __forceinline__ bool rng_full(const Rng& r)
     return (r.x1 == r.x0 + 1) & (r.y1 == r.y0 + 1) & (r.z1 == r.z0 + 1);
 }
 
-// A full 2x2x2 block packed in 31 bits (base voxel, 10 bits per axis, G <= 1024);
-// 0 marks "not a full block".
-__device__ __forceinline__ uint32_t pack_block(const Rng& r)
-{
-    return rng_full(r) ? (0x80000000u | (uint32_t)r.x0 | ((uint32_t)r.y0 << 10) | ((uint32_t)r.z0 << 20)) : 0u;
-}
-
-__device__ __forceinline__ Rng unpack_block(uint32_t p)
-{
-    Rng r;
-    r.x0 = (int)(p & 1023u);
-    r.y0 = (int)((p >> 10) & 1023u);
-    r.z0 = (int)((p >> 20) & 1023u);
-    r.x1 = r.x0 + 1;
-    r.y1 = r.y0 + 1;
-    r.z1 = r.z0 + 1;
-    return r;
-}
-
 // Friction blend (compute.comp:296-297): (1 - mu) * v + mu * v_grid.
 __device__ __forceinline__ f3 friction(f3 v, f3 gv, float mu, float omu) { return add(smul(omu, v), smul(mu, gv)); }
 
@@ -83,6 +64,30 @@ __device__ __forceinline__ bool in_win(const Rng& r, const Win& w)
 {
     return (r.x0 >= w.x0) & (r.x1 < w.x0 + w.ex) & (r.y0 >= w.y0) & (r.y1 < w.y0 + w.ey) & (r.z0 >= w.z0) &
            (r.z1 < w.z0 + w.ez);
+}
+
+// A point whose whole 2x2x2 block lies in a window: its lower corner relative
+// to the window, and the corner's grid coordinates as floats.  (NaN converts
+// to 0, which is the range the shader's int() gives it; its weights are 0.)
+struct Loc {
+    uint32_t x, y, z;
+    f3 lo;
+};
+
+__device__ __forceinline__ bool locate(f3 q, const Win& w, Loc& l)
+{
+    l.lo = mk(floorf(q.x), floorf(q.y), floorf(q.z));
+    l.x = (uint32_t)(sat_i32(l.lo.x) - w.x0);
+    l.y = (uint32_t)(sat_i32(l.lo.y) - w.y0);
+    l.z = (uint32_t)(sat_i32(l.lo.z) - w.z0);
+    // a window reaches at most to the grid's last voxel, so both corners are in the grid
+    return (l.x < (uint32_t)(w.ex - 1)) & (l.y < (uint32_t)(w.ey - 1)) & (l.z < (uint32_t)(w.ez - 1));
+}
+
+// Linear index of a located point's lower corner (24-bit factors: full-rate multiplies).
+__device__ __forceinline__ uint32_t loc_index(const Loc& l, const Win& w)
+{
+    return __umul24(__umul24(l.z, (uint32_t)w.ey) + l.y, (uint32_t)w.ex) + l.x;
 }
 
 __device__ __forceinline__ int win_index(const Win& w, int a, int b, int c)
@@ -120,16 +125,16 @@ __device__ __forceinline__ void gather_cell(f3& gv, float4 c, float w)
     gv = add(gv, smul(t, mk(c.x, c.y, c.z)));
 }
 
-__device__ __forceinline__ float wgt(float q, int a) { return clamp01(1.0f - fabsf(q - (float)a)); }
+__device__ __forceinline__ float wgt(float q, float a) { return clamp01(1.0f - fabsf(q - a)); }
 
-// Full 2x2x2 block inside an LDS window of float cells.
-__device__ __forceinline__ f3 gather_block(const float4* win, const Win& wd, const Rng& r, f3 q)
+// Full 2x2x2 block inside a window of float cells.
+__device__ __forceinline__ f3 gather_block(const float4* win, const Win& wd, const Loc& l, f3 q)
 {
-    const float wx0 = wgt(q.x, r.x0), wx1 = wgt(q.x, r.x1);
-    const float wy0 = wgt(q.y, r.y0), wy1 = wgt(q.y, r.y1);
-    const float wz0 = wgt(q.z, r.z0), wz1 = wgt(q.z, r.z1);
+    const float wx0 = wgt(q.x, l.lo.x), wx1 = wgt(q.x, l.lo.x + 1.0f);
+    const float wy0 = wgt(q.y, l.lo.y), wy1 = wgt(q.y, l.lo.y + 1.0f);
+    const float wz0 = wgt(q.z, l.lo.z), wz1 = wgt(q.z, l.lo.z + 1.0f);
     const int sy = wd.ex, sz = wd.ex * wd.ey;
-    const float4* b = win + win_index(wd, r.x0, r.y0, r.z0);
+    const float4* b = win + loc_index(l, wd);
     const float4 c000 = b[0], c001 = b[sz], c010 = b[sy], c011 = b[sy + sz];
     const float4 c100 = b[1], c101 = b[1 + sz], c110 = b[1 + sy], c111 = b[1 + sy + sz];
     f3 gv = mk(0.0f, 0.0f, 0.0f);
@@ -159,13 +164,13 @@ __device__ __forceinline__ f3 gather_any_src(const float4* win, const Win& wd, c
     f3 gv = mk(0.0f, 0.0f, 0.0f);
 #pragma unroll 1
     for (int a = r.x0; a <= r.x1; ++a) {
-        const float wxa = wgt(q.x, a);
+        const float wxa = wgt(q.x, (float)a);
 #pragma unroll 1
         for (int b = r.y0; b <= r.y1; ++b) {
-            const float wxy = wxa * wgt(q.y, b);
+            const float wxy = wxa * wgt(q.y, (float)b);
 #pragma unroll 1
             for (int c = r.z0; c <= r.z1; ++c) {
-                const float w = wxy * wgt(q.z, c);
+                const float w = wxy * wgt(q.z, (float)c);
                 float4 cell;
                 if (LDS)
                     cell = win[win_index(wd, a, b, c)];
@@ -184,6 +189,17 @@ __device__ __forceinline__ f3 gather_any(const float4* win, const Win& wd, bool 
     return lds ? gather_any_src<true>(win, wd, g, r, q, G) : gather_any_src<false>(win, wd, g, r, q, G);
 }
 
+// From the global float grid: the whole grid as the window.
+__device__ __forceinline__ f3 gather_grid(const float4* __restrict__ g, int G, f3 q)
+{
+    const Win all{0, 0, 0, G, G, G};
+    Loc l;
+    if (locate(q, all, l)) return gather_block(g, all, l, q);
+    const Rng rg = point_range(q, G);
+    if (rng_empty(rg)) return mk(0.0f, 0.0f, 0.0f);
+    return gather_any_src<false>(nullptr, all, g, rg, q, G);
+}
+
 // ---------------------------------------------------------------------------
 // Splat.  Contributions int(SCALE*(w*v)) and int(SCALE*w) (compute.comp:241-248)
 // accumulate in an LDS window holding `nc` copies of every voxel (nc a power
@@ -191,11 +207,18 @@ __device__ __forceinline__ f3 gather_any(const float4* win, const Win& wd, bool 
 // lane l adds into copy l & (nc-1).  Hair is dense: tens of lanes of one
 // wavefront land in the same voxel block, and same-address LDS atomics
 // serialise, so a small box is spread over copies that the dump sums.
-// A copy is 16 B:  u64 (vx << 32 | density), u32 vy, u32 vz.
+// An entry is a u64 (vx << 32 | density), a u32 vy and a u32 vz, each in a
+// plane of its own: the lanes of one atomic then spread over all LDS banks
+// (16 B entries put every vy on an eighth of them).
 // Density addends are in [0, 1e6] and one window holds at most kW*(kL+1)
 // points, so the low word never carries into vx: both sums are exact mod 2^32.
 // ---------------------------------------------------------------------------
-constexpr int kMaxCopies = 16;
+#ifndef HS_COPIES
+#define HS_COPIES 16
+#endif
+constexpr int kMaxCopies = HS_COPIES;
+constexpr uint32_t kWinY = kWinCells * 8;       // byte offsets of the vy and vz planes
+constexpr uint32_t kWinZ = kWinCells * 8 + kWinCells * 4;
 
 // Where a lane's splat goes: its copy and the order it visits the corners of
 // its 2x2x2 block in (lanes that share a copy take different orders).  Copy k of
@@ -225,34 +248,56 @@ __device__ __forceinline__ void splat_cell(unsigned char* win, int e, float w, f
     const uint32_t iy = (uint32_t)sat_i32(SCALE * wv.y);
     const uint32_t iz = (uint32_t)sat_i32(SCALE * wv.z);
     const uint32_t id = (uint32_t)sat_i32(SCALE * w);
-    unsigned char* cellp = win + 16 * e;
-    atomicAdd(reinterpret_cast<unsigned long long*>(cellp), ((unsigned long long)ix << 32) | id);
-    atomicAdd(reinterpret_cast<uint32_t*>(cellp + 8), iy);
-    atomicAdd(reinterpret_cast<uint32_t*>(cellp + 12), iz);
+    atomicAdd(reinterpret_cast<unsigned long long*>(win + 8 * e), ((unsigned long long)ix << 32) | id);
+    atomicAdd(reinterpret_cast<uint32_t*>(win + kWinY + 4 * e), iy);
+    atomicAdd(reinterpret_cast<uint32_t*>(win + kWinZ + 4 * e), iz);
 }
 
-// Sum of window voxel w's copies as a GridCell (vx, vy, vz, density).
-__device__ __forceinline__ int4 splat_sum(const int4* win, int w, const SplatLane& sl)
+// Sum of window voxel w's NC copies as a GridCell (vx, vy, vz, density).  The
+// copies of one voxel are consecutive: read 16 B at a time, four copies in flight.
+template <int NC>
+__device__ __forceinline__ int4 splat_sum(const int4* win, int w)
 {
+    const unsigned char* b = reinterpret_cast<const unsigned char*>(win);
     uint64_t A = 0;
     uint32_t sy = 0, sz = 0;
-    for (int k = 0; k < sl.nc; ++k) {
-        const int4 raw = win[w * sl.nc + k];
-        A += ((uint64_t)(uint32_t)raw.y << 32) | (uint32_t)raw.x;
-        sy += (uint32_t)raw.z;
-        sz += (uint32_t)raw.w;
+    if constexpr (NC == 1) {
+        A = *reinterpret_cast<const uint64_t*>(b + 8 * w);
+        sy = *reinterpret_cast<const uint32_t*>(b + kWinY + 4 * w);
+        sz = *reinterpret_cast<const uint32_t*>(b + kWinZ + 4 * w);
+    } else {
+        if constexpr (NC == 2) {
+            const ulonglong2 A2 = *reinterpret_cast<const ulonglong2*>(b + 16 * w);
+            const uint2 y = *reinterpret_cast<const uint2*>(b + kWinY + 8 * w);
+            const uint2 z = *reinterpret_cast<const uint2*>(b + kWinZ + 8 * w);
+            A = A2.x + A2.y;
+            sy = y.x + y.y;
+            sz = z.x + z.y;
+        } else {
+            const ulonglong2* pa = reinterpret_cast<const ulonglong2*>(b + 8 * NC * w);
+            const uint4* py = reinterpret_cast<const uint4*>(b + kWinY + 4 * NC * w);
+            const uint4* pz = reinterpret_cast<const uint4*>(b + kWinZ + 4 * NC * w);
+#pragma unroll 1
+            for (int k = 0; k < NC / 4; ++k) {
+                const ulonglong2 a0 = pa[2 * k], a1 = pa[2 * k + 1];
+                const uint4 y = py[k], z = pz[k];
+                A += (a0.x + a0.y) + (a1.x + a1.y);
+                sy += (y.x + y.y) + (y.z + y.w);
+                sz += (z.x + z.y) + (z.z + z.w);
+            }
+        }
     }
     return make_int4((int)(uint32_t)(A >> 32), (int)sy, (int)sz, (int)(uint32_t)A);
 }
 
 // Full 2x2x2 block inside the LDS window.
-__device__ __forceinline__ void splat_block(int4* win, const Win& wd, const Rng& r, f3 q, f3 v, const SplatLane& sl)
+__device__ __forceinline__ void splat_block(int4* win, const Win& wd, const Loc& l, f3 q, f3 v, const SplatLane& sl)
 {
-    const float wx0 = wgt(q.x, r.x0), wx1 = wgt(q.x, r.x1);
-    const float wy0 = wgt(q.y, r.y0), wy1 = wgt(q.y, r.y1);
-    const float wz0 = wgt(q.z, r.z0), wz1 = wgt(q.z, r.z1);
+    const float wx0 = wgt(q.x, l.lo.x), wx1 = wgt(q.x, l.lo.x + 1.0f);
+    const float wy0 = wgt(q.y, l.lo.y), wy1 = wgt(q.y, l.lo.y + 1.0f);
+    const float wz0 = wgt(q.z, l.lo.z), wz1 = wgt(q.z, l.lo.z + 1.0f);
     const int sx = sl.nc, sy = sx * wd.ex, sz = sy * wd.ey;
-    const int e0 = splat_entry(win_index(wd, r.x0, r.y0, r.z0), sl);
+    const int e0 = (int)__umul24(loc_index(l, wd), (uint32_t)sl.nc) + sl.slot;
     unsigned char* wb = reinterpret_cast<unsigned char*>(win);
     // Lanes that share a copy visit the corners in different orders (step i
     // takes corner i ^ rot), so lanes of one voxel block hit different cells
@@ -282,13 +327,13 @@ __device__ __forceinline__ void splat_any(int4* win, const Win& wd, bool lds, co
     const float SCALE = 1000000.0f;
 #pragma unroll 1
     for (int a = r.x0; a <= r.x1; ++a) {
-        const float wxa = wgt(q.x, a);
+        const float wxa = wgt(q.x, (float)a);
 #pragma unroll 1
         for (int b = r.y0; b <= r.y1; ++b) {
-            const float wxy = wxa * wgt(q.y, b);
+            const float wxy = wxa * wgt(q.y, (float)b);
 #pragma unroll 1
             for (int c = r.z0; c <= r.z1; ++c) {
-                const float w = wxy * wgt(q.z, c);
+                const float w = wxy * wgt(q.z, (float)c);
                 if (lds) {
                     splat_cell(reinterpret_cast<unsigned char*>(win), splat_entry(win_index(wd, a, b, c), sl), w, v);
                 } else {
@@ -326,9 +371,9 @@ __device__ __forceinline__ f3 force_at(f3 x, f3 fs, const StepArgs& a, float4 mf
         const float d2 = dot(dv, dv);
         // d2 < sphere_r2 is exactly sqrt(d2) < sphere_r
         if (d2 < a.sphere_r2) {
-            const float dist = sqrtf(d2);
+            const float dist = sqrt_rn(d2);
             const float d = a.sphere_r - dist;
-            const f3 n = muls(dv, 1.0f / dist);
+            const f3 n = muls(dv, rcp_sqrt(d2));
             acc = add(acc, smul(a.k * d, n));
             hits = 1;
         }
@@ -358,7 +403,9 @@ __device__ __forceinline__ f3 force_at(f3 x, f3 fs, const StepArgs& a, float4 mf
         }
     }
     f3 force = fs;
-    if (hits > 0) {
+    if (hits == 1) {
+        force = add(force, acc);  // divided by 1
+    } else if (COL != 0 && hits > 1) {
         const float m = (float)hits;
         force = add(force, mk(acc.x / m, acc.y / m, acc.z / m));
     }
@@ -393,9 +440,6 @@ __device__ __forceinline__ GridWork global_grid(const GridWork& in)
     w.brick_list = global_ptr(in.brick_list);
     w.brick_nz = global_ptr(in.brick_nz);
     w.near_limit = global_ptr(in.near_limit);
-    w.dlist = global_ptr(in.dlist);
-    w.dclaim = global_ptr(in.dclaim);
-    w.dbox = global_ptr(in.dbox);
     return w;
 }
 

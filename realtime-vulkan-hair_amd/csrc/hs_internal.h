@@ -33,8 +33,7 @@ struct DevHeap {
 
 // Shape-derived sizes of one groom's device state.
 // Strand planes padded to Sp slots; the grid workspace holds the pool slots,
-// descriptors and deferred-list entries of the tile shape with the most
-// workgroup-segments (nws_cap).
+// descriptors of the tile shape with the most workgroup-segments (nws_cap).
 struct Layout {
     uint32_t Sp, nws_cap;
     uint64_t pool_cap, desc_cap;
@@ -69,7 +68,6 @@ struct Groom {
     bool pending = false;
     float pend_mu = 0.0f, pend_omu = 1.0f;
     uint32_t parity = 0;           // pool/counter half the next splat writes
-    uint32_t steps = 0;            // steps launched (the kernels' list tag)
     int last_shape = -1;           // tile shape of the last splat step (its gbox layout)
     uint64_t bytes = 0;            // size of `block`
 };

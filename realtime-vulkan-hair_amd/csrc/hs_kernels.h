@@ -31,7 +31,9 @@ constexpr uint32_t kBricksPerWG = 4;
 constexpr uint32_t kMaxColliders = 8;
 constexpr uint32_t kDescInts = 8;     // partial-box descriptor: lo xyz, ext xyz, pool offset, pad
 constexpr uint32_t kBrickList = 2048;  // box indices kept per reduce brick (more: it scans every box)
-constexpr int kDBoxInts = 12;          // deferred segment: box lo xyz, hi xyz, chunk extents y z, counts y z, pad
+// bits of counters[parity][2]
+constexpr uint32_t kFellBack = 1;      // a box larger than any window, or a full pool
+constexpr uint32_t kOverflowUsed = 2;  // the overflow grid holds sums of this step
 constexpr uint32_t kSlotCells = HS_WINDOW_CELLS;  // pool cells a workgroup-segment owns for its
                                                  // first box (a whole splat window)
 
@@ -41,7 +43,7 @@ struct GridWork {
     float4* grid_f;       // G^3 (float(vx), float(vy), float(vz), density > 0 ? 1/float(density) : 0)
     int4* pool;           // partial boxes written by the step kernel, [2][pool_cap]
     int* desc;            // partial-box descriptors, [2][desc_cap][kDescInts]
-    uint32_t* counters;   // [2][4]: shared cells used, shared boxes used, fallback flag, deferred entries
+    uint32_t* counters;   // [2][4]: shared cells used, shared boxes used, overflow bits, segments of several windows
     int4* overflow;       // G^3 int4 atomic fallback when the pool is full (normally zero)
     int* gbox;            // [nwg][nseg][6] voxel box each workgroup-segment touched last step (laid
                           // out for the last step's tile shape)
@@ -49,17 +51,11 @@ struct GridWork {
     uint32_t* brick_list; // [2][nbricks][kBrickList] indices of the boxes overlapping a brick
     uint32_t* brick_nz;   // [nbricks] 1 when the brick's grid cells are not all zero
     unsigned long long* near_limit;  // (cell, step) pairs with a component >= 2^30 in magnitude
-    // workgroup-segments whose box needs several windows, splatted chunk by
-    // chunk by any workgroup of the groom that is done with its own strands
-    unsigned long long* dlist;  // [2][nws_cap] step tag (28 bits) | chunks (12) | workgroup-segment (24)
-    uint32_t* dclaim;           // [2][nws_cap] chunks taken of each list entry
-    int* dbox;                  // [nws_cap][kDBoxInts] box and chunking of a deferred segment
     // pool / descriptors per parity: first each workgroup-segment's own slot
     // (kSlotCells cells, descriptor index = its number), then a shared part
     // taken with atomics; pool_cap / desc_cap count both
     uint32_t pool_cap, desc_cap;
     uint32_t nws;            // workgroup-segments of the launch's tile shape: owners of the slots
-    uint32_t nws_cap;        // the most any tile shape has: the stride of dlist / dclaim halves
     uint32_t nbx, nby, nbz;  // reduce bricks per axis
 };
 
@@ -96,8 +92,6 @@ struct StepArgs {
     // voxel grid (compute.comp:9-11, 204-206)
     GridWork gw;
     uint32_t G, parity;   // parity selects pool/counter half written by this launch
-    uint32_t tag;         // 1 + steps of this groom launched before, mod 2^28 - 1 (tells deferred-list
-                          // entries apart; never 0, the value of a list slot not written yet)
     float ox, oy, oz, inv_h;
     float mu_prev, omu_prev;  // friction of the previous step and 1 - friction
     // step constants

@@ -9,12 +9,12 @@
 //
 // One step = two kernels.
 //  k_step   (one workgroup per kW strands, hs_step.hip) walks each strand root
-//           to tip in segments of kL points held in registers.  Per segment:
+//           to tip in segments of kL points.  Per segment:
 //             P: per point, friction with the previous step's voxel window
 //                staged in LDS (compute.comp:257-298), force and predicted
 //                position (compute.comp:150-187), all points independent;
-//             F: follow-the-leader, damped velocity, DFTL (compute.comp:
-//                190-215), the root-to-tip chain;
+//             F: follow-the-leader (compute.comp:190-192), the root-to-tip chain;
+//             V: damped velocity, correction, DFTL (compute.comp:195-215);
 //             S: trilinear fixed-point splat (compute.comp:217-252) of the
 //                points whose velocity is final into an LDS window, dumped as
 //                a dense partial box to a pool.
@@ -285,11 +285,8 @@ __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uin
     const uint32_t nlisted = gw.brick_cnt[parity * nbr + brick];
     if (lane == 0) gw.brick_cnt[(parity ^ 1u) * nbr + brick] = 0;  // for the step after next
     if (reset_counters) {
-        // the next step's counters, and the chunk claims of the previous
-        // step's deferred list (the next step uses the same half)
+        // the next step's counters
         uint32_t* nxt = gw.counters + (parity ^ 1u) * 4;
-        const uint32_t nd = nxt[3];
-        for (uint32_t i = lane; i < nd && i < gw.nws_cap; i += 64) gw.dclaim[(size_t)(parity ^ 1u) * gw.nws_cap + i] = 0;
         if (lane == 0) {
             nxt[0] = 0;
             nxt[1] = 0;
@@ -458,14 +455,7 @@ __global__ __launch_bounds__(kTileThreads) void k_unpack(float4* __restrict__ ao
                 if (g && i >= 1) {
                     const f3 pp = mk(pos[o], pos[plane + o], pos[2 * plane + o]);
                     const f3 q = grid_coord(pp, mk(ox, oy, oz), inv_h);
-                    const Rng rg = point_range(q, (int)G);
-                    f3 gv = mk(0.0f, 0.0f, 0.0f);
-                    const int Gi = (int)G;
-                    if (rng_full(rg))
-                        gv = gather_block(g, Win{0, 0, 0, Gi, Gi, Gi}, rg, q);  // the whole grid as the window
-                    else if (!rng_empty(rg))
-                        gv = gather_any_src<false>(nullptr, Win{0, 0, 0, 0, 0, 0}, g, rg, q, Gi);
-                    v = friction(v, gv, mu, omu);
+                    v = friction(v, gather_grid(g, (int)G, q), mu, omu);
                 }
                 val = make_float4(v.x, v.y, v.z, 0.0f);
             } else if (corr) {
