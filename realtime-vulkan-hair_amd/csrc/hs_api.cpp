@@ -763,7 +763,7 @@ int groom_build(const hs_groom_desc* d, const float* aos, hipStream_t st, DevHea
     return HS_OK;
 }
 
-hipError_t groom_unpack(const Groom& g, float* aos_dev, hipStream_t st)
+hipError_t groom_unpack(const Groom& g, float* aos_dev, hipStream_t st, uint32_t* rec_dev)
 {
     hs::UnpackGrid ug;
     const hs::UnpackGrid* pug = nullptr;
@@ -778,7 +778,7 @@ hipError_t groom_unpack(const Groom& g, float* aos_dev, hipStream_t st)
         ug.omu = g.pend_omu;
         pug = &ug;
     }
-    return hs::launch_unpack(aos_dev, g.perm, g.S, g.N, g.L.Sp, g.pos, g.vel, g.corr,
+    return hs::launch_unpack(aos_dev, rec_dev, g.perm, g.S, g.N, g.L.Sp, g.pos, g.vel, g.corr,
                              pug, st);
 }
 
@@ -1285,8 +1285,7 @@ int hs_export_strands(hs_ctx* c, uint32_t id, float* aos_dev, uint32_t* ind_dev)
     Groom* g = find(c, id);
     if (!g) return fail(c, HS_ERR_NOT_FOUND, "hs_export_strands: unknown groom");
     HS_TRY(c, hipSetDevice(c->device));
-    HS_TRY(c, groom_unpack(*g, aos_dev, c->stream));
-    if (ind_dev) HS_TRY(c, hs::launch_indirect(ind_dev, g->S, c->stream));
+    HS_TRY(c, groom_unpack(*g, aos_dev, c->stream, ind_dev));
     return HS_OK;
 }
 

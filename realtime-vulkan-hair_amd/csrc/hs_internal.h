@@ -87,8 +87,9 @@ int groom_build(const hs_groom_desc* d, const float* aos, hipStream_t st, DevHea
 void groom_release(Groom& g);
 
 // Reference-layout copy of the groom (pending friction applied) into device
-// memory `aos_dev` (48*S*N bytes), on stream `st`.
-hipError_t groom_unpack(const Groom& g, float* aos_dev, hipStream_t st);
+// memory `aos_dev` (48*S*N bytes), and the indirect draw record into `rec_dev`
+// (16 B) when given, on stream `st`.
+hipError_t groom_unpack(const Groom& g, float* aos_dev, hipStream_t st, uint32_t* rec_dev = nullptr);
 
 // A mesh collider on the device (hs_mesh_create).
 struct Mesh {

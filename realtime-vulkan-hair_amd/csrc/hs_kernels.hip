@@ -421,54 +421,90 @@ __global__ void k_pack(const float4* __restrict__ aos, const uint32_t* __restric
 // in LDS, reading each point plane with consecutive lanes on consecutive
 // slots, then writes every strand's block contiguously in caller order.
 // Rows are padded to N+1 entries against LDS bank conflicts.
-constexpr uint32_t kTileF4 = 2048;  // float4 entries of the LDS tile (32 KiB)
 constexpr uint32_t kTileThreads = 256;
+
+// Strand slots per output tile, for `rows` LDS rows of N + 1 float4 per strand:
+// a power of two, at most 32 (128 B of a point plane per read) and 54 KB of
+// LDS (three workgroups per CU), down to 8 (which any N <= 256 fits in 66 KB)
+// while the launch has fewer than two workgroups per CU.
+static uint32_t tile_strands(uint32_t S, uint32_t N, uint32_t rows)
+{
+    uint32_t ts = 32;
+    while (ts > 8 && (ts * (N + 1) * rows * 16 > 54u << 10 || (S + ts - 1) / ts < 512)) ts /= 2;
+    return ts;
+}
+
+// Written once and not read here: kept out of the caches the planes and the
+// grid are read through.
+__device__ __forceinline__ void st_stream(float4* p, float4 v)
+{
+    using v4 = float __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(v4{v.x, v.y, v.z, v.w}, reinterpret_cast<v4*>(p));
+}
 
 // SoA -> AoS (Strand layout); when `g` (the float cells of the last step's
 // grid) is given, applies the pending grid friction to velocities of points
-// 1..N-1 (compute.comp:257-298) on the way.
+// 1..N-1 (compute.comp:257-298) on the way.  Block 0 writes the indirect draw
+// record {S, 1, 0, 0} (the shader's count, compute.comp:302) when asked to.
+// Positions and velocities go through LDS together, one barrier for both (a
+// pass per array read the positions twice and waited three times); the
+// correction rows, zero unless kept, follow.  Bound by HBM: 24 B read and 48 B
+// written per point; 100,000 x 32 73.6 -> 44.2 us (5.2 TB/s), a groom of about
+// 1,000 x 16 15.7 -> 4.9 us (narrower tiles: more workgroups), and the draw
+// record no longer takes a launch of its own.
+template <bool CORR>
 __global__ __launch_bounds__(kTileThreads) void k_unpack(float4* __restrict__ aos, const uint32_t* __restrict__ perm,
                                                          uint32_t S, uint32_t N, uint32_t Sp,
                                                          const float* __restrict__ pos, const float* __restrict__ vel,
                                                          const float* __restrict__ corr, const float4* __restrict__ g,
                                                          uint32_t G, float ox, float oy, float oz, float inv_h,
-                                                         float mu, float omu, uint32_t ts)
+                                                         float mu, float omu, uint32_t ts, uint32_t* __restrict__ rec)
 {
-    __shared__ float4 tile[kTileF4];
+    extern __shared__ float4 tile[];
+    if (rec && blockIdx.x == 0 && threadIdx.x < 4) rec[threadIdx.x] = threadIdx.x == 0 ? S : (threadIdx.x == 1 ? 1u : 0u);
     const uint32_t p0 = blockIdx.x * ts;
     const uint32_t ns = min(ts, S - p0);
     const uint32_t row = N + 1;
     const size_t plane = (size_t)N * Sp;
-    // ts (N + 1) <= kTileF4: indices and divisors stay below 2^16, where the
-    // reciprocal multiply divides exactly
-    const uint32_t m_ts = div_magic(ts), m_n = div_magic(N);
-    for (uint32_t arr = 0; arr < 3; ++arr) {
-        for (uint32_t e = threadIdx.x; e < ts * N; e += kTileThreads) {
-            const uint32_t i = div_small(e, ts, m_ts), pl = e - i * ts;
-            if (pl >= ns) continue;
-            const size_t o = (size_t)i * Sp + p0 + pl;
-            float4 val = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (arr == 0) {
-                val = make_float4(pos[o], pos[plane + o], pos[2 * plane + o], 1.0f);
-            } else if (arr == 1) {
-                f3 v = mk(vel[o], vel[plane + o], vel[2 * plane + o]);
-                if (g && i >= 1) {
-                    const f3 pp = mk(pos[o], pos[plane + o], pos[2 * plane + o]);
-                    const f3 q = grid_coord(pp, mk(ox, oy, oz), inv_h);
-                    v = friction(v, gather_grid(g, (int)G, q), mu, omu);
-                }
-                val = make_float4(v.x, v.y, v.z, 0.0f);
-            } else if (corr) {
-                val = make_float4(corr[o], corr[plane + o], corr[2 * plane + o], 0.0f);
+    float4* tv = tile + ts * row;
+    float4* tc = tv + ts * row;
+    // ts is a power of two, and ts * N stays below 2^16, where the reciprocal
+    // multiply divides exactly
+    const uint32_t lts = 31 - __clz(ts);
+    const uint32_t pl = threadIdx.x & (ts - 1);
+    if (pl < ns) {
+        // two points at a time, their loads in flight together
+        constexpr uint32_t kU = 2;
+        const uint32_t di = kTileThreads >> lts;
+        for (uint32_t i0 = threadIdx.x >> lts; i0 < N; i0 += kU * di) {
+            f3 x[kU], v[kU], c[kU];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; ++u) {
+                const size_t o = (size_t)min(i0 + u * di, N - 1) * Sp + p0 + pl;
+                x[u] = mk(pos[o], pos[plane + o], pos[2 * plane + o]);
+                v[u] = mk(vel[o], vel[plane + o], vel[2 * plane + o]);
+                if (CORR) c[u] = mk(corr[o], corr[plane + o], corr[2 * plane + o]);
             }
-            tile[pl * row + i] = val;
+#pragma unroll
+            for (uint32_t u = 0; u < kU; ++u) {
+                const uint32_t i = i0 + u * di;
+                if (i >= N) break;
+                if (g && i >= 1)
+                    v[u] = friction(v[u], gather_grid(g, (int)G, grid_coord(x[u], mk(ox, oy, oz), inv_h)), mu, omu);
+                tile[pl * row + i] = make_float4(x[u].x, x[u].y, x[u].z, 1.0f);
+                tv[pl * row + i] = make_float4(v[u].x, v[u].y, v[u].z, 0.0f);
+                if (CORR) tc[pl * row + i] = make_float4(c[u].x, c[u].y, c[u].z, 0.0f);
+            }
         }
-        __syncthreads();
-        for (uint32_t e = threadIdx.x; e < ns * N; e += kTileThreads) {
-            const uint32_t pl = div_small(e, N, m_n), i = e - pl * N;
-            aos[((size_t)perm[p0 + pl] * 3 + arr) * N + i] = tile[pl * row + i];
-        }
-        __syncthreads();
+    }
+    __syncthreads();
+    const uint32_t m_n = div_magic(N);
+    for (uint32_t e = threadIdx.x; e < ns * N; e += kTileThreads) {
+        const uint32_t sl = div_small(e, N, m_n), i = e - sl * N;
+        float4* out = aos + (size_t)perm[p0 + sl] * 3 * N + i;
+        st_stream(out, tile[sl * row + i]);
+        st_stream(out + N, tv[sl * row + i]);
+        st_stream(out + 2 * N, CORR ? tc[sl * row + i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     }
 }
 
@@ -482,7 +518,8 @@ __global__ __launch_bounds__(kTileThreads) void k_unpack(float4* __restrict__ ao
 // (1/3)((v3 - v1)/2); de Casteljau with mix(a,b,t) = a*(1-t) + b*t.  At v = 1
 // the shader would read one point past the strand; here it is the tip
 // (last segment, t = 1).  Positions staged per tile as in k_unpack; samples
-// written strand by strand.
+// written strand by strand.  Bound by HBM: 100,000 x 32, 64 samples, 38.6 ->
+// 25.7 us (5.5 TB/s) with reciprocal divides and streaming stores.
 __device__ __forceinline__ f3 mix3(f3 a, f3 b, float t)
 {
     const float u = 1.0f - t;
@@ -494,20 +531,29 @@ __global__ __launch_bounds__(kTileThreads) void k_resample(const float* __restri
                                                            uint32_t Sp, uint32_t M, float4* __restrict__ out,
                                                            uint32_t ts)
 {
-    __shared__ float4 tile[kTileF4];
+    extern __shared__ float4 tile[];
     const uint32_t p0 = blockIdx.x * ts;
     const uint32_t ns = min(ts, S - p0);
     const uint32_t row = N + 1;
     const size_t plane = (size_t)N * Sp;
-    for (uint32_t e = threadIdx.x; e < ts * N; e += kTileThreads) {
-        const uint32_t pl = e % ts, i = e / ts;
-        if (pl >= ns) continue;
-        const size_t o = (size_t)i * Sp + p0 + pl;
-        tile[pl * row + i] = make_float4(pos[o], pos[plane + o], pos[2 * plane + o], 0.0f);
+    const uint32_t lts = 31 - __clz(ts);
+    {
+        const uint32_t pl = threadIdx.x & (ts - 1);
+        if (pl < ns) {
+            for (uint32_t i = threadIdx.x >> lts; i < N; i += kTileThreads >> lts) {
+                const size_t o = (size_t)i * Sp + p0 + pl;
+                tile[pl * row + i] = make_float4(pos[o], pos[plane + o], pos[2 * plane + o], 0.0f);
+            }
+        }
     }
     __syncthreads();
+    // sample e of the tile: strand e / M, sample e % M; ns * M < 2^16 when M
+    // is below 2048, where the reciprocal multiply divides exactly
+    const bool small = M < 2048;
+    const uint32_t m_m = div_magic(small ? M : 1);
     for (uint32_t e = threadIdx.x; e < ns * M; e += kTileThreads) {
-        const uint32_t pl = e / M, j = e % M;
+        const uint32_t pl = small ? div_small(e, M, m_m) : e / M;
+        const uint32_t j = e - pl * M;
         const float4* T = tile + pl * row;
         auto P = [&](uint32_t i) {
             const float4 v = T[i];
@@ -533,17 +579,8 @@ __global__ __launch_bounds__(kTileThreads) void k_resample(const float* __restri
         const f3 b01 = mix3(b0, b1, t), b11 = mix3(b1, b2, t), b21 = mix3(b2, b3, t);
         const f3 b02 = mix3(b01, b11, t), b12 = mix3(b11, b21, t);
         const f3 c = mix3(b02, b12, t);
-        out[(size_t)perm[p0 + pl] * M + j] = make_float4(c.x, c.y, c.z, 1.0f);
+        st_stream(out + (size_t)perm[p0 + pl] * M + j, make_float4(c.x, c.y, c.z, 1.0f));
     }
-}
-
-// Strand slots per output tile: whole padded rows of N + 1 entries.
-static uint32_t tile_strands(uint32_t N) { return max(1u, min(64u, kTileF4 / (N + 1))); }
-
-// The indirect draw record the shader's count produces (compute.comp:302).
-__global__ void k_indirect(uint32_t* __restrict__ rec, uint32_t S)
-{
-    if (threadIdx.x < 4) rec[threadIdx.x] = threadIdx.x == 0 ? S : (threadIdx.x == 1 ? 1u : 0u);
 }
 
 // ---------------------------------------------------------------------------
@@ -596,31 +633,23 @@ hipError_t launch_pack(const float* aos_dev, const uint32_t* perm, uint32_t S, u
 hipError_t launch_resample(const float* pos, const uint32_t* perm, uint32_t S, uint32_t N, uint32_t Sp, uint32_t M,
                            float* out_dev, hipStream_t st)
 {
-    if (N < 2 || M < 2 || N + 1 > kTileF4) return hipErrorInvalidValue;
-    const uint32_t ts = tile_strands(N);
-    hipLaunchKernelGGL(k_resample, dim3((S + ts - 1) / ts), dim3(kTileThreads), 0, st, pos, perm, S, N, Sp, M,
+    if (N < 2 || M < 2 || N > 256) return hipErrorInvalidValue;
+    const uint32_t ts = tile_strands(S, N, 1);
+    hipLaunchKernelGGL(k_resample, dim3((S + ts - 1) / ts), dim3(kTileThreads), ts * (N + 1) * 16, st, pos, perm, S, N, Sp, M,
                        reinterpret_cast<float4*>(out_dev), ts);
     return hipGetLastError();
 }
 
-hipError_t launch_indirect(uint32_t* rec_dev, uint32_t S, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_indirect, dim3(1), dim3(64), 0, st, rec_dev, S);
-    return hipGetLastError();
-}
-
-hipError_t launch_unpack(float* aos_dev, const uint32_t* perm, uint32_t S, uint32_t N, uint32_t Sp,
+hipError_t launch_unpack(float* aos_dev, uint32_t* rec_dev, const uint32_t* perm, uint32_t S, uint32_t N, uint32_t Sp,
                          const float* pos, const float* vel, const float* corr, const UnpackGrid* g, hipStream_t st)
 {
-    if (N + 1 > kTileF4) return hipErrorInvalidValue;
-    const uint32_t ts = tile_strands(N);
-    const dim3 grid((S + ts - 1) / ts), block(kTileThreads);
-    if (g)
-        hipLaunchKernelGGL(k_unpack, grid, block, 0, st, reinterpret_cast<float4*>(aos_dev), perm, S, N, Sp, pos, vel,
-                           corr, g->grid, g->G, g->ox, g->oy, g->oz, g->inv_h, g->mu, g->omu, ts);
-    else
-        hipLaunchKernelGGL(k_unpack, grid, block, 0, st, reinterpret_cast<float4*>(aos_dev), perm, S, N, Sp, pos, vel,
-                           corr, (const float4*)nullptr, 0u, 0.f, 0.f, 0.f, 0.f, 0.f, 1.f, ts);
+    if (N > 256) return hipErrorInvalidValue;
+    const uint32_t rows = corr ? 3 : 2;
+    const uint32_t ts = tile_strands(S, N, rows);
+    const UnpackGrid u = g ? *g : UnpackGrid{nullptr, 0, 0.f, 0.f, 0.f, 0.f, 0.f, 1.f};
+    hipLaunchKernelGGL((corr ? k_unpack<true> : k_unpack<false>), dim3((S + ts - 1) / ts), dim3(kTileThreads),
+                       ts * (N + 1) * rows * 16, st, reinterpret_cast<float4*>(aos_dev), perm, S, N, Sp, pos, vel, corr,
+                       u.grid, u.G, u.ox, u.oy, u.oz, u.inv_h, u.mu, u.omu, ts, rec_dev);
     return hipGetLastError();
 }
 

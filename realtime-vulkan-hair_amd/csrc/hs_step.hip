@@ -8,12 +8,13 @@
 // chains.  Now only the follow-the-leader recurrence is walked one lane per
 // strand (28 instructions a point, a seventh of the step); the rest has four
 // threads per strand at 128 x 16 and two at the 256-strand shapes, 4
-// wavefronts per SIMD.  Measured (us, before -> after): 100,000 x 32, 128 x 16
-// 104 -> 82; 20,000 x 32 94 -> 47; eight grooms of 512-2048 strands in one
-// launch 170 -> 64; 1,000,000 x 64 with the head mesh, 256 x 8, settled hair
-// 2,560 -> 1,560.  It issues 27.6M vector instructions at 100,000 x 32 (47 us
-// at one per 4 cycles); the rest is LDS time (same-address atomics of dense
-// hair) and barriers.
+// wavefronts per SIMD.  Measured (before -> after, exports included): 8 steps
+// of 100,000 x 32, 128 x 16, 1,029 -> 838 us; 4 steps of 37,501 x 57, 256 x 8,
+// 857 -> 555 us; one step of eight grooms of 512-2,048 strands 300 -> 208 us;
+// 4 steps of 1,000,000 x 64 with the head mesh, 256 x 8, 19.3 -> 16.1 ms.  It
+// issues 27.6M vector instructions a step at 100,000 x 32 (47 us at one per 4
+// cycles); the rest is LDS time (same-address atomics of dense hair),
+// barriers and load latency.
 //
 // This file is compiled once per shape the library offers, each build in its own
 // namespace (HS_SHAPE_NS) with HS_TILE_STRANDS / HS_TILE_POINTS set; results
