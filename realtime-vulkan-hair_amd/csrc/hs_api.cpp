@@ -784,6 +784,60 @@ hipError_t groom_unpack(const Groom& g, float* aos_dev, hipStream_t st, uint32_t
 
 }  // namespace hsi
 
+namespace {
+
+// Drops the list entries that no point of their cell can have as its nearest
+// triangle (on the device), and moves the mesh to a block of the new size.
+// Where there is no memory for that, the lists stay as they are: the search's
+// result is the same.
+int prune_mesh(hs_ctx* c, hsi::Mesh& m, std::vector<uint32_t>& starts, float margin, uint64_t tri_bytes, uint64_t start_bytes)
+{
+    const size_t ncell = starts.size() - 1;
+    const uint32_t entries = starts[ncell];
+    if (entries == 0) return HS_OK;
+    uint8_t* work = nullptr;  // counts, then keep flags
+    uint8_t* block = nullptr;
+    const uint64_t count_bytes = round_up(ncell * 4, 256);
+    auto done = [&](hipError_t e) {
+        (void)hipFree(work);
+        if (e == hipSuccess) return (int)HS_OK;
+        (void)hipFree(block);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            return (int)HS_OK;
+        }
+        return hip_fail(c, e, "hs_mesh_create: candidate lists");
+    };
+    hipError_t e = hipMalloc((void**)&work, count_bytes + entries);
+    if (e != hipSuccess) return done(e);
+    uint32_t* count = reinterpret_cast<uint32_t*>(work);
+    uint8_t* keep = work + count_bytes;
+    e = hs::launch_mesh_prune(m.args, (uint32_t)ncell, margin, keep, count, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(starts.data() + 1, count, ncell * 4, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return done(e);
+    for (size_t k = 1; k <= ncell; ++k) starts[k] += starts[k - 1];
+    const uint64_t bytes = tri_bytes + start_bytes + round_up(std::max<uint64_t>(starts[ncell], 1) * 48, 256);
+    e = hipMalloc((void**)&block, bytes);
+    if (e != hipSuccess) return done(e);
+    uint32_t* to = reinterpret_cast<uint32_t*>(block + tri_bytes);
+    float4* recs = reinterpret_cast<float4*>(block + tri_bytes + start_bytes);
+    e = hipMemcpyAsync(block, m.block, tri_bytes, hipMemcpyDeviceToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(to, starts.data(), starts.size() * 4, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hs::launch_mesh_compact(m.args, (uint32_t)ncell, keep, to, recs, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return done(e);
+    (void)hipFree(m.block);
+    m.block = block;
+    m.bytes = bytes;
+    m.args.tris = reinterpret_cast<const float4*>(block);
+    m.args.cell_start = to;
+    m.args.cell_recs = recs;
+    return done(hipSuccess);
+}
+
+}  // namespace
+
 extern "C" {
 
 int hs_groom_create(hs_ctx* c, const hs_groom_desc* d, const float* aos, uint32_t* id)
@@ -851,6 +905,11 @@ int hs_mesh_create(hs_ctx* c, const float* v, uint32_t nv, const uint32_t* t, ui
     a.dy = b.dim[1];
     a.dz = b.dim[2];
     a.margin2 = d->margin * d->margin;
+    int rc = prune_mesh(c, m, b.cell_start, d->margin, tri_bytes, start_bytes);
+    if (rc != HS_OK) {
+        (void)hipFree(m.block);
+        return rc;
+    }
     const uint32_t mid = c->next_mesh++;
     c->meshes[mid] = m;
     c->bytes += m.bytes;

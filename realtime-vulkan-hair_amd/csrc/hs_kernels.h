@@ -154,6 +154,12 @@ inline hipError_t launch_step_batch(int shape, const StepArgs* args_dev, const u
     }
 }
 hipError_t launch_reduce(const GridWork& gw, uint32_t G, uint32_t parity, hipStream_t st);
+// Pruning of a new mesh's candidate lists: keep[entry] and each cell's count
+// of kept entries; then the kept records, at the starts `to`, into `out`.
+hipError_t launch_mesh_prune(const MeshArgs& M, uint32_t ncell, float margin, uint8_t* keep, uint32_t* count,
+                             hipStream_t st);
+hipError_t launch_mesh_compact(const MeshArgs& M, uint32_t ncell, const uint8_t* keep, const uint32_t* to, float4* out,
+                               hipStream_t st);
 // Mesh pass: mesh contact of every stored position of `a` into a.mesh_f
 // (N * Sp float4).  Runs before a step kernel that reads it.
 hipError_t launch_mesh_force(const StepArgs& a, hipStream_t st);
