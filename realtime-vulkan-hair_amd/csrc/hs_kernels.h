@@ -25,9 +25,8 @@ constexpr uint32_t kMaxTileStrands = 256;
 #define HS_WINDOW_CELLS 2048
 #endif
 constexpr uint32_t kWinCells = HS_WINDOW_CELLS;  // LDS window of one workgroup, 16 B entries
-// reduce kernel: bricks of kBX x kBY x kBZ voxels, one wavefront each
+// reduce kernel: bricks of kBX x kBY x kBZ voxels, one workgroup each
 constexpr uint32_t kBX = 8, kBY = 4, kBZ = 2;
-constexpr uint32_t kBricksPerWG = 4;
 constexpr uint32_t kMaxColliders = 8;
 constexpr uint32_t kDescInts = 8;     // partial-box descriptor: lo xyz, ext xyz, pool offset, pad
 constexpr uint32_t kBrickList = 2048;  // box indices kept per reduce brick (more: it scans every box)

@@ -18,7 +18,7 @@
 //             S: trilinear fixed-point splat (compute.comp:217-252) of the
 //                points whose velocity is final into an LDS window, dumped as
 //                a dense partial box to a pool.
-//  k_reduce (one workgroup per 8^3 voxel brick) sums every partial box that
+//  k_reduce (one workgroup per 64-voxel brick) sums every partial box that
 //           overlaps its brick and writes the step's grid: the GridCell ints
 //           and the float cells the next step's G phase reads.  It writes every
 //           voxel, which also clears the grid (the vkCmdFillBuffer of
@@ -326,10 +326,18 @@ __global__ __launch_bounds__(256) void k_mesh_force_batch(const StepArgs* __rest
 // ---------------------------------------------------------------------------
 // Reduce: partial boxes -> grid (GridCell ints + float cells); clears the grid.
 // ---------------------------------------------------------------------------
-// One wavefront per brick of kBX x kBY x kBZ = 64 voxels, one voxel per lane:
-// each lane sums its voxel over the boxes listed for the brick in registers
-// (wrapping int32 adds, order independent), kInFlight boxes per round.
-constexpr uint32_t kReduceThreads = 64 * kBricksPerWG;
+// One workgroup per brick of kBX x kBY x kBZ = 64 voxels, one voxel per lane:
+// each lane sums its voxel over its wavefront's share of the boxes listed for
+// the brick in registers (wrapping int32 adds, order independent).
+// Wavefronts that share a brick's boxes, kInFlight at a time.  A brick's walk
+// is a chain of dependent loads (count, list, descriptors, cells), 30 boxes
+// long on average and hundreds where hair is dense, and the launch lasts as
+// long as its longest chains: four wavefronts per brick take 8 steps at
+// 100,000 x 32 from 791 to 710 us a call, against 737 with two (and 708 with
+// eight of 8).  A batch has bricks enough to hide the chains and pays for
+// wavefronts that find nothing listed: 256 grooms x 8 steps 9.67 -> 9.29 ms
+// with two, 10.06 with four.
+constexpr uint32_t kReduceWaves = 4, kReduceWavesBatch = 2;
 constexpr uint32_t kInFlight = 16;
 static_assert(kBX * kBY * kBZ == 64, "one voxel per lane");
 
@@ -361,71 +369,64 @@ __device__ __forceinline__ void add4(uint4& acc, int4 v)
 
 __device__ __forceinline__ bool near_limit(int v) { return v >= (1 << 30) || v <= -(1 << 30); }
 
+template <uint32_t kWaves>
 __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uint32_t parity, uint32_t brick,
                                              bool reset_counters)
 {
+    __shared__ uint4 part[kWaves - 1][64];
     const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t nbr = gw.nbx * gw.nby * gw.nbz;
+    const uint32_t* ctr = gw.counters + parity * 4;
+    const bool ovf = ctr[2] != 0;
+    const uint32_t nlisted = gw.brick_cnt[parity * nbr + brick];
+    if (threadIdx.x == 0) gw.brick_cnt[(parity ^ 1u) * nbr + brick] = 0;  // for the step after next
+    if (reset_counters && threadIdx.x < 4) gw.counters[(parity ^ 1u) * 4 + threadIdx.x] = 0;  // the next step's
+    // nothing listed, no overflow, and zero already: the brick stays as it is
+    if (nlisted == 0 && !ovf && gw.brick_nz[brick] == 0) return;
+
     const uint32_t bx = brick % gw.nbx, by = (brick / gw.nbx) % gw.nby, bz = brick / (gw.nbx * gw.nby);
     const int cx = (int)(bx * kBX + (lane % kBX)), cy = (int)(by * kBY + (lane / kBX) % kBY),
               cz = (int)(bz * kBZ + lane / (kBX * kBY));
     const bool inside = cx < (int)G && cy < (int)G && cz < (int)G;
-    const uint32_t* ctr = gw.counters + parity * 4;
-    const bool ovf = ctr[2] != 0;
-    const uint32_t nlisted = gw.brick_cnt[parity * nbr + brick];
-    if (lane == 0) gw.brick_cnt[(parity ^ 1u) * nbr + brick] = 0;  // for the step after next
-    if (reset_counters) {
-        // the next step's counters
-        uint32_t* nxt = gw.counters + (parity ^ 1u) * 4;
-        if (lane == 0) {
-            nxt[0] = 0;
-            nxt[1] = 0;
-            nxt[2] = 0;
-            nxt[3] = 0;
-        }
-    }
-    // nothing listed, no overflow, and zero already: the brick stays as it is
-    if (nlisted == 0 && !ovf && gw.brick_nz[brick] == 0) return;
-
     const int* desc = gw.desc + (size_t)parity * gw.desc_cap * kDescInts;
     const int4* pool = gw.pool + (size_t)parity * gw.pool_cap;
     uint4 acc = make_uint4(0, 0, 0, 0);
     // a compile-time capacity: with a run-time one this kernel measured 1.8x slower
     if (nlisted <= kBrickList) {
         const uint32_t* bl = gw.brick_list + ((size_t)parity * nbr + brick) * kBrickList;
-        for (uint32_t base = 0; base < nlisted; base += 64) {
-            // lane l fetches box base+l's descriptor: one dependent load chain per 64 boxes
-            const uint32_t m = min(64u, nlisted - base);
+        // the wavefronts take kInFlight boxes in turn
+        for (uint32_t base = wave * kInFlight; base < nlisted; base += kWaves * kInFlight) {
+            // lane l fetches box base+l's descriptor, then every lane walks
+            // the boxes, all their cell loads in flight
+            const uint32_t m = min(kInFlight, nlisted - base);
             int4 d0 = make_int4(0, 0, 0, 0), d1 = make_int4(0, 0, 0, 0);
             if (lane < m) {
                 const int4* dp = reinterpret_cast<const int4*>(desc + (size_t)bl[base + lane] * kDescInts);
                 d0 = dp[0];
                 d1 = dp[1];
             }
-            // then every lane walks the boxes, kInFlight cell loads at a time
-            for (uint32_t j = 0; j < m; j += kInFlight) {
-                int4 v[kInFlight];
+            int4 v[kInFlight];
 #pragma unroll
-                for (uint32_t u = 0; u < kInFlight; ++u) {
-                    v[u] = make_int4(0, 0, 0, 0);
-                    if (j + u < m) {
-                        const int src = (int)(j + u);
-                        const BoxRef b{__builtin_amdgcn_readlane(d0.x, src), __builtin_amdgcn_readlane(d0.y, src),
-                                       __builtin_amdgcn_readlane(d0.z, src), __builtin_amdgcn_readlane(d0.w, src),
-                                       __builtin_amdgcn_readlane(d1.x, src), __builtin_amdgcn_readlane(d1.y, src),
-                                       __builtin_amdgcn_readlane(d1.z, src)};
-                        v[u] = box_cell(b, pool, cx, cy, cz);
-                    }
+            for (uint32_t u = 0; u < kInFlight; ++u) {
+                v[u] = make_int4(0, 0, 0, 0);
+                if (u < m) {
+                    const int src = (int)u;
+                    const BoxRef b{__builtin_amdgcn_readlane(d0.x, src), __builtin_amdgcn_readlane(d0.y, src),
+                                   __builtin_amdgcn_readlane(d0.z, src), __builtin_amdgcn_readlane(d0.w, src),
+                                   __builtin_amdgcn_readlane(d1.x, src), __builtin_amdgcn_readlane(d1.y, src),
+                                   __builtin_amdgcn_readlane(d1.z, src)};
+                    v[u] = box_cell(b, pool, cx, cy, cz);
                 }
-#pragma unroll
-                for (uint32_t u = 0; u < kInFlight; ++u) add4(acc, v[u]);
             }
+#pragma unroll
+            for (uint32_t u = 0; u < kInFlight; ++u) add4(acc, v[u]);
         }
     } else {
         // the brick's list overflowed: scan every box of the step
         const uint32_t ndesc = min(gw.nws + ctr[1], gw.desc_cap);
         const int x0 = (int)(bx * kBX), y0 = (int)(by * kBY), z0 = (int)(bz * kBZ);
-        for (uint32_t i = 0; i < ndesc; ++i) {
+        for (uint32_t i = wave; i < ndesc; i += kWaves) {
             const BoxRef b = box_ref(desc + (size_t)i * kDescInts);
             if (b.ex <= 0 || b.x0 > x0 + (int)kBX - 1 || b.x0 + b.ex <= x0 || b.y0 > y0 + (int)kBY - 1 ||
                 b.y0 + b.ey <= y0 || b.z0 > z0 + (int)kBZ - 1 || b.z0 + b.ez <= z0)
@@ -433,6 +434,19 @@ __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uin
             add4(acc, box_cell(b, pool, cx, cy, cz));
         }
     }
+    // join the wavefronts' sums (one wavefront is enough for a short list)
+    if (nlisted > kInFlight) {
+        if (wave > 0) part[wave - 1][lane] = acc;
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (uint32_t w = 0; w + 1 < kWaves; ++w) {
+                const uint4 p = part[w][lane];
+                add4(acc, make_int4((int)p.x, (int)p.y, (int)p.z, (int)p.w));
+            }
+        }
+    }
+    if (wave > 0) return;
     bool nz = false, near = false;
     if (inside) {
         const uint32_t gi = (uint32_t)cx + (uint32_t)cy * G + (uint32_t)cz * G * G;
@@ -454,26 +468,19 @@ __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uin
     }
 }
 
-__global__ __launch_bounds__(kReduceThreads) void k_reduce(GridWork gw, uint32_t G, uint32_t parity)
+__global__ __launch_bounds__(64 * kReduceWaves) void k_reduce(GridWork gw, uint32_t G, uint32_t parity)
 {
-    const uint32_t brick = blockIdx.x * kBricksPerWG + (threadIdx.x >> 6);
-    if (brick >= gw.nbx * gw.nby * gw.nbz) return;
-    reduce_brick(gw, G, parity, brick, brick == 0);
+    reduce_brick<kReduceWaves>(gw, G, parity, blockIdx.x, blockIdx.x == 0);
 }
 
 // Many grooms: brick_start[g] is the first global brick of groom g.
-__global__ __launch_bounds__(kReduceThreads) void k_reduce_batch(const StepArgs* __restrict__ args,
+__global__ __launch_bounds__(64 * kReduceWavesBatch) void k_reduce_batch(const StepArgs* __restrict__ args,
                                                                  const uint32_t* __restrict__ brick_start,
                                                                  uint32_t ngroom)
 {
-    const uint32_t total = brick_start[ngroom];
-    // one brick per wavefront: the index is wave-uniform, and saying so keeps
-    // the groom lookup and its arguments in scalar registers
-    const uint32_t gb = __builtin_amdgcn_readfirstlane(blockIdx.x * kBricksPerWG + (threadIdx.x >> 6));
-    if (gb >= total) return;
-    const uint32_t g = __builtin_amdgcn_readfirstlane(find_groom(brick_start, ngroom, gb));
-    const uint32_t b = gb - brick_start[g];
-    reduce_brick(global_grid(args[g].gw), args[g].G, args[g].parity, b, b == 0);
+    const uint32_t g = __builtin_amdgcn_readfirstlane(find_groom(brick_start, ngroom, blockIdx.x));
+    const uint32_t b = blockIdx.x - brick_start[g];
+    reduce_brick<kReduceWavesBatch>(global_grid(args[g].gw), args[g].G, args[g].parity, b, b == 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -679,8 +686,7 @@ __global__ __launch_bounds__(kTileThreads) void k_resample(const float* __restri
 hipError_t launch_reduce_batch(const StepArgs* args_dev, const uint32_t* brick_start_dev, uint32_t ngroom,
                                uint32_t total_bricks, hipStream_t st)
 {
-    const uint32_t blocks = (total_bricks + kBricksPerWG - 1) / kBricksPerWG;
-    hipLaunchKernelGGL(k_reduce_batch, dim3(blocks), dim3(kReduceThreads), 0, st, args_dev, brick_start_dev, ngroom);
+    hipLaunchKernelGGL(k_reduce_batch, dim3(total_bricks), dim3(64 * kReduceWavesBatch), 0, st, args_dev, brick_start_dev, ngroom);
     return hipGetLastError();
 }
 
@@ -722,8 +728,7 @@ hipError_t launch_reduce(const GridWork& gw, uint32_t G, uint32_t parity, hipStr
 {
     (void)G;
     const uint32_t nbr = gw.nbx * gw.nby * gw.nbz;
-    hipLaunchKernelGGL(k_reduce, dim3((nbr + kBricksPerWG - 1) / kBricksPerWG), dim3(kReduceThreads), 0, st, gw, G,
-                       parity);
+    hipLaunchKernelGGL(k_reduce, dim3(nbr), dim3(64 * kReduceWaves), 0, st, gw, G, parity);
     return hipGetLastError();
 }
 
