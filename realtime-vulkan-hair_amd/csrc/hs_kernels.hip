@@ -338,6 +338,10 @@ __global__ __launch_bounds__(256) void k_mesh_force_batch(const StepArgs* __rest
 // wavefronts that find nothing listed: 256 grooms x 8 steps 9.67 -> 9.29 ms
 // with two, 10.06 with four.
 constexpr uint32_t kReduceWaves = 4, kReduceWavesBatch = 2;
+// A groom of at most this many workgroup-segments lists few boxes per brick,
+// and most of its launch is wavefronts that find an empty brick: one wavefront
+// per brick.
+constexpr uint32_t kShortLists = 32;
 constexpr uint32_t kInFlight = 16;
 static_assert(kBX * kBY * kBZ == 64, "one voxel per lane");
 
@@ -373,15 +377,15 @@ template <uint32_t kWaves>
 __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uint32_t parity, uint32_t brick,
                                              bool reset_counters)
 {
-    __shared__ uint4 part[kWaves - 1][64];
+    __shared__ uint4 part[kWaves > 1 ? kWaves - 1 : 1][64];
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave = kWaves > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const uint32_t nbr = gw.nbx * gw.nby * gw.nbz;
     const uint32_t* ctr = gw.counters + parity * 4;
     const bool ovf = ctr[2] != 0;
     const uint32_t nlisted = gw.brick_cnt[parity * nbr + brick];
-    if (threadIdx.x == 0) gw.brick_cnt[(parity ^ 1u) * nbr + brick] = 0;  // for the step after next
-    if (reset_counters && threadIdx.x < 4) gw.counters[(parity ^ 1u) * 4 + threadIdx.x] = 0;  // the next step's
+    if (wave == 0 && lane == 0) gw.brick_cnt[(parity ^ 1u) * nbr + brick] = 0;  // for the step after next
+    if (reset_counters && wave == 0 && lane < 4) gw.counters[(parity ^ 1u) * 4 + lane] = 0;  // the next step's
     // nothing listed, no overflow, and zero already: the brick stays as it is
     if (nlisted == 0 && !ovf && gw.brick_nz[brick] == 0) return;
 
@@ -435,7 +439,7 @@ __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uin
         }
     }
     // join the wavefronts' sums (one wavefront is enough for a short list)
-    if (nlisted > kInFlight) {
+    if (kWaves > 1 && nlisted > kInFlight) {
         if (wave > 0) part[wave - 1][lane] = acc;
         __syncthreads();
         if (wave == 0) {
@@ -471,6 +475,13 @@ __device__ __forceinline__ void reduce_brick(const GridWork& gw, uint32_t G, uin
 __global__ __launch_bounds__(64 * kReduceWaves) void k_reduce(GridWork gw, uint32_t G, uint32_t parity)
 {
     reduce_brick<kReduceWaves>(gw, G, parity, blockIdx.x, blockIdx.x == 0);
+}
+
+// Short lists only: a wavefront per brick, four bricks per workgroup.
+__global__ __launch_bounds__(256) void k_reduce_short(GridWork gw, uint32_t G, uint32_t parity)
+{
+    const uint32_t brick = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (brick < gw.nbx * gw.nby * gw.nbz) reduce_brick<1>(gw, G, parity, brick, brick == 0);
 }
 
 // Many grooms: brick_start[g] is the first global brick of groom g.
@@ -728,7 +739,10 @@ hipError_t launch_reduce(const GridWork& gw, uint32_t G, uint32_t parity, hipStr
 {
     (void)G;
     const uint32_t nbr = gw.nbx * gw.nby * gw.nbz;
-    hipLaunchKernelGGL(k_reduce, dim3(nbr), dim3(64 * kReduceWaves), 0, st, gw, G, parity);
+    if (gw.nws <= kShortLists)
+        hipLaunchKernelGGL(k_reduce_short, dim3((nbr + 3) / 4), dim3(256), 0, st, gw, G, parity);
+    else
+        hipLaunchKernelGGL(k_reduce, dim3(nbr), dim3(64 * kReduceWaves), 0, st, gw, G, parity);
     return hipGetLastError();
 }
 
