@@ -532,22 +532,29 @@ __global__ void k_pack(const float4* __restrict__ aos, const uint32_t* __restric
 constexpr uint32_t kTileThreads = 256;
 
 // Strand slots per output tile, for `rows` LDS rows of N + 1 float4 per strand:
-// a power of two, at most 32 (128 B of a point plane per read) and 54 KB of
+// a power of two, at most 32 (128 B of a point plane per read; 64 for strands
+// too short to give the threads work) and 54 KB of
 // LDS (three workgroups per CU), down to 8 (which any N <= 256 fits in 66 KB)
 // while the launch has fewer than two workgroups per CU.
 static uint32_t tile_strands(uint32_t S, uint32_t N, uint32_t rows)
 {
-    uint32_t ts = 32;
+    uint32_t ts = N <= 8 ? 64 : 32;
     while (ts > 8 && (ts * (N + 1) * rows * 16 > 54u << 10 || (S + ts - 1) / ts < 512)) ts /= 2;
     return ts;
 }
 
 // Written once and not read here: kept out of the caches the planes and the
-// grid are read through.
-__device__ __forceinline__ void st_stream(float4* p, float4 v)
+// grid are read through, where a strand's row is whole cache lines.  Shorter
+// rows need the cache to join them into lines (200,000 x 2 exported each step:
+// 31 us streamed, 20 through the cache; 100,000 x 5: 29 and 21).
+constexpr uint32_t kStreamRow = 16;  // entries (256 B)
+__device__ __forceinline__ void st_out(float4* p, float4 v, bool stream)
 {
     using v4 = float __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(v4{v.x, v.y, v.z, v.w}, reinterpret_cast<v4*>(p));
+    if (stream)
+        __builtin_nontemporal_store(v4{v.x, v.y, v.z, v.w}, reinterpret_cast<v4*>(p));
+    else
+        *p = v;
 }
 
 // SoA -> AoS (Strand layout); when `g` (the float cells of the last step's
@@ -607,12 +614,13 @@ __global__ __launch_bounds__(kTileThreads) void k_unpack(float4* __restrict__ ao
     }
     __syncthreads();
     const uint32_t m_n = div_magic(N);
+    const bool stream = N >= kStreamRow;
     for (uint32_t e = threadIdx.x; e < ns * N; e += kTileThreads) {
         const uint32_t sl = div_small(e, N, m_n), i = e - sl * N;
         float4* out = aos + (size_t)perm[p0 + sl] * 3 * N + i;
-        st_stream(out, tile[sl * row + i]);
-        st_stream(out + N, tv[sl * row + i]);
-        st_stream(out + 2 * N, CORR ? tc[sl * row + i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+        st_out(out, tile[sl * row + i], stream);
+        st_out(out + N, tv[sl * row + i], stream);
+        st_out(out + 2 * N, CORR ? tc[sl * row + i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f), stream);
     }
 }
 
@@ -655,10 +663,11 @@ __global__ __launch_bounds__(kTileThreads) void k_resample(const float* __restri
         }
     }
     __syncthreads();
-    // sample e of the tile: strand e / M, sample e % M; ns * M < 2^16 when M
-    // is below 2048, where the reciprocal multiply divides exactly
-    const bool small = M < 2048;
+    // sample e of the tile: strand e / M, sample e % M; below 2^16 the
+    // reciprocal multiply divides exactly
+    const bool small = M < 65536 / ts;
     const uint32_t m_m = div_magic(small ? M : 1);
+    const bool stream = M >= kStreamRow;
     for (uint32_t e = threadIdx.x; e < ns * M; e += kTileThreads) {
         const uint32_t pl = small ? div_small(e, M, m_m) : e / M;
         const uint32_t j = e - pl * M;
@@ -687,7 +696,7 @@ __global__ __launch_bounds__(kTileThreads) void k_resample(const float* __restri
         const f3 b01 = mix3(b0, b1, t), b11 = mix3(b1, b2, t), b21 = mix3(b2, b3, t);
         const f3 b02 = mix3(b01, b11, t), b12 = mix3(b11, b21, t);
         const f3 c = mix3(b02, b12, t);
-        st_stream(out + (size_t)perm[p0 + pl] * M + j, make_float4(c.x, c.y, c.z, 1.0f));
+        st_out(out + (size_t)perm[p0 + pl] * M + j, make_float4(c.x, c.y, c.z, 1.0f), stream);
     }
 }
 

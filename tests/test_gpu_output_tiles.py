@@ -26,7 +26,7 @@ def _stepped(ctx, wl, keep):
 
 
 @pytest.mark.parametrize("keep", [False, True])
-@pytest.mark.parametrize("S,N", [(1, 2), (31, 52), (33, 53), (17, 107), (9, 108), (7, 256), (40, 256), (16500, 3)])
+@pytest.mark.parametrize("S,N", [(1, 2), (31, 52), (33, 53), (17, 107), (9, 108), (7, 256), (40, 256), (16500, 3), (140000, 2)])
 def test_export_tiles(ctx, S, N, keep):
     wl = scenes.plain_100k(S=S, N=N, G=16)
     gpu, ref = _stepped(ctx, wl, keep)
@@ -47,7 +47,7 @@ def test_export_tiles(ctx, S, N, keep):
         gpu.destroy()
 
 
-@pytest.mark.parametrize("S,N,M", [(33, 16, 2047), (33, 16, 2048), (3, 256, 5000), (1, 2, 2), (16500, 3, 4)])
+@pytest.mark.parametrize("S,N,M", [(33, 16, 8191), (33, 16, 8192), (140000, 2, 5), (3, 256, 5000), (1, 2, 2), (16500, 3, 4)])
 def test_resample_tiles(ctx, S, N, M):
     wl = scenes.plain_100k(S=S, N=N, G=16)
     gpu, ref = _stepped(ctx, wl, False)

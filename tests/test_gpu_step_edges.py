@@ -3,12 +3,12 @@ threads has edges: strands that end on a segment's or a thread's last point,
 one past it, and one before it, for every tile shape; workgroups with a single
 strand or one short of full; boxes of many splat windows and of more than the
 kernel splats through windows.  Bitwise against ref32."""
-import numpy as np
 import pytest
 
 import hairsim
+import oracle
 from hairsim import scenes
-from helpers import run_parity
+from helpers import assert_bitwise, gpu_params, make_gpu_groom, oracle_params, run_parity
 
 pytestmark = pytest.mark.gpu
 
@@ -53,6 +53,27 @@ def test_corrections_and_plain_steps_at_edges(ctx):
     """Kept corrections, and steps without the grid (no splat, no gather)."""
     wl = scenes.plain_100k(S=130, N=17, G=16)
     run_parity(ctx, wl, 3, keep_corrections=True)
-    for N in (2, 16, 17, 18, 33):
+    for N in (2, 5, 9, 10, 16, 17, 18, 33):  # up to 9 points take the 256 x 8 kernel whatever the tile
         run_parity(ctx, scenes.plain_1k(S=130, N=N), 3, keep_corrections=True)
-    assert np.isfinite(wl.grooms[0].strands).all()
+
+
+@pytest.mark.parametrize("N", [2, 9, 10])
+def test_grid_switched_on_and_off(ctx, N):
+    """Steps with and without the grid in turn: the latter may run another
+    shape, which must not be taken for the layout of the last splat's boxes."""
+    wl = scenes.plain_100k(S=300, N=N, G=16)
+    g = wl.grooms[0]
+    gpu = make_gpu_groom(ctx, wl)
+    ref, grid = g.strands.copy(), None
+    try:
+        for k, on in enumerate([True, False, False, True, True, False, True]):
+            c = [scenes.sphere_collider(wl.sphere(k))]
+            gpu.step(wl.dt, float(wl.time(k)), c, gpu_params(wl, k, hair_hair=on))
+            grid = oracle.step32(oracle_params(wl, k, hair_hair=on), ref, N, grid)
+        out = gpu.read()[0].reshape(-1, 3, N, 4).copy()
+        want = ref.reshape(-1, 3, N, 4).copy()
+        out[:, 2] = 0
+        want[:, 2] = 0
+        assert_bitwise(out, want, f"N={N}", N)
+    finally:
+        gpu.destroy()
