@@ -188,7 +188,7 @@ def tune_tile(ctx, hairsim, scenes, wl, mesh_id, warmup):
 
 def tile_record(tile, tuned_ms):
     return {"gather_cells": tile[0], "splat_cells": tile[1], "xcd_order": tile[2], "strands_per_workgroup": tile[3],
-            "points_per_segment": tile[4], "strands_per_wavefront": 64, "autotuned_ms_per_step": tuned_ms}
+            "points_per_segment": tile[4], "strands_per_wavefront": tile[3] // 8, "autotuned_ms_per_step": tuned_ms}
 
 
 def bench_single(args, hairsim, scenes, wl):

@@ -32,13 +32,13 @@ __device__ __forceinline__ float dot(f3 a, f3 b) { return (a.x * b.x + a.y * b.y
 
 // Correctly rounded square root and reciprocal in short sequences: the
 // hardware estimate, then one refinement whose residual is exact in a fused
-// multiply-add.  For x in [2^-100, 2^100] nothing over- or underflows on the
+// multiply-add.  For x in [2^-100, 2^100) nothing over- or underflows on the
 // way, and there both give the bits of sqrtf(x) and 1.0f / x for every float
 // (all 1,677,721,600 of them compared on gfx950); other values take the
 // compiler's general sequences, which are twice as long.
 __device__ __forceinline__ bool mid_range(float x)
 {
-    return __float_as_uint(x) - ((127u - 100u) << 23) <= (200u << 23);
+    return __float_as_uint(x) - ((127u - 100u) << 23) < (200u << 23);
 }
 __device__ __forceinline__ float sqrt_rn(float x)
 {

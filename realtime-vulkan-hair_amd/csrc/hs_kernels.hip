@@ -25,7 +25,7 @@
 //           Renderer.cpp:2063).
 // The step is skewed: the friction of step k is applied by k_step of step
 // k+1 (or by the read-back kernel).  Per point the operations and their order
-// are those of the unskewed shader, so results are bit-identical; integer
+// are those of the unskewed shader, so results are bit-identical.
 //
 // This file holds the shape-independent kernels (mesh pass, reduce, layout
 // conversion, resampling); the step kernels are in hs_step.hip, built once
